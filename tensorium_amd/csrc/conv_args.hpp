@@ -181,6 +181,9 @@ __device__ inline void conv_store_buf(const ConvArgs& a, const f32x16 (&acc)[FM]
   const int rowBase = static_cast<int>(m0w) + 4 * h;  // row of element (i = 0, r = 0)
   const bool allRows = m0w + FM * 32 <= a.F;          // wave-uniform
   auto rowOk = [&](int c) { return allRows || rowBase + c < F; };
+  // row c of the block for a scalar offset: no row past the last (kOOB)
+  const int lastRow = __builtin_amdgcn_readfirstlane(max(F - 1 - static_cast<int>(m0w), 0));
+  auto row = [&](int c) { return static_cast<uint32_t>(min(c, lastRow)); };
   if (a.splits > 1) {
     const uint32_t N = static_cast<uint32_t>(a.g.N);
     const int64_t slice = a.F * a.g.N;
@@ -194,7 +197,7 @@ __device__ inline void conv_store_buf(const ConvArgs& a, const f32x16 (&acc)[FM]
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int c = i * 32 + 8 * (r >> 2) + (r & 3);
-          buf_st1s(pr, acc[i][j][r], rowOk(c) ? vo : kOOB, static_cast<uint32_t>(c) * N * 4u);
+          buf_st1s(pr, acc[i][j][r], rowOk(c) ? vo : kOOB, row(c) * N * 4u);
         }
     }
     return;
@@ -230,7 +233,7 @@ __device__ inline void conv_store_buf(const ConvArgs& a, const f32x16 (&acc)[FM]
     vOut[j] = sel_off(okN, (b * static_cast<uint32_t>(a.outBatchStride) + rowOff) * 4u);
     vRes[j] = sel_off(okN, (b * static_cast<uint32_t>(a.rBatchStride) + rowOff) * 4u);
   }
-  auto so = [&](int i, int r) { return static_cast<uint32_t>(i * 32 + 8 * (r >> 2) + (r & 3)) * OHW * 4u; };
+  auto so = [&](int i, int r) { return row(i * 32 + 8 * (r >> 2) + (r & 3)) * OHW * 4u; };
   // The activation and the residual are wave-uniform: each combination gets
   // its own straight-line code, and every residual load is issued before the
   // first store (a store may alias a later residual element, so interleaved
@@ -312,6 +315,9 @@ __device__ __attribute__((always_inline)) inline void conv_store_nhwc(const Conv
   const int rowBase = static_cast<int>(m0w) + 4 * h;  // pixel of element (i = 0, r = 0)
   const bool allRows = m0w + FM * 32 <= M;
   auto rowOk = [&](int c) { return allRows || rowBase + c < M; };
+  // pixel c of the block for a scalar offset: none past the last (kOOB)
+  const int lastRow = __builtin_amdgcn_readfirstlane(max(static_cast<int>(M) - 1 - static_cast<int>(m0w), 0));
+  auto row = [&](int c) { return static_cast<uint32_t>(min(c, lastRow)); };
   const uint32_t op4 = static_cast<uint32_t>(a.outPix) * 4u, rp4 = static_cast<uint32_t>(a.resPix) * 4u;
   const __amdgpu_buffer_rsrc_t outR = make_rsrc(a.out, a.outBytes);
   const __amdgpu_buffer_rsrc_t resR = make_rsrc(a.res, a.resBytes);
@@ -357,7 +363,7 @@ __device__ __attribute__((always_inline)) inline void conv_store_nhwc(const Conv
               y[e] = yolo_entry(v[e], entry);
               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v[e]), outR,
                                                     rowOk(c0 + e) ? vOut[j] : kOOB,
-                                                    static_cast<uint32_t>(c0 + e) * op4, 0);
+                                                    row(c0 + e) * op4, 0);
             }
             const uint32_t m = static_cast<uint32_t>(rowBase + c0);
             if (a.yoloVec) {  // m % 4 == 0 and M % 4 == 0: the 4 pixels are in range together, in one image
@@ -410,7 +416,7 @@ __device__ __attribute__((always_inline)) inline void conv_store_nhwc(const Conv
         for (int j = 0; j < FN; ++j)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            rv[i][j][r] = buf_ld1s(resR, rowOk(rc(i, r)) ? vRes[j] : kOOB, static_cast<uint32_t>(rc(i, r)) * rp4);
+            rv[i][j][r] = buf_ld1s(resR, rowOk(rc(i, r)) ? vRes[j] : kOOB, row(rc(i, r)) * rp4);
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -420,7 +426,7 @@ __device__ __attribute__((always_inline)) inline void conv_store_nhwc(const Conv
         for (int r = 0; r < 16; ++r) {
           float v = apply_act(acc[i][j][r] + bias[j], ACT);
           if constexpr (RES) v = v + rv[i][j][r];
-          buf_st1s(outR, v, rowOk(rc(i, r)) ? vOut[j] : kOOB, static_cast<uint32_t>(rc(i, r)) * op4);
+          buf_st1s(outR, v, rowOk(rc(i, r)) ? vOut[j] : kOOB, row(rc(i, r)) * op4);
         }
   };
   using Leaky = std::integral_constant<int, TNH_AC_LEAKY>;

@@ -39,7 +39,7 @@ struct GatherCols {
   uint32_t colOff;        // bytes to (image, iy0, ix0), modulo 2^32
   uint32_t yMask, xMask;  // window rows and columns inside the image
   GatherDiv div;
-  int q0, K, kw, W, inner;
+  int q0, K, kw, W, C, inner;
   bool tap;
   uint32_t HW4;
   int ldsOff[NQ];
@@ -51,6 +51,7 @@ struct GatherCols {
     K = static_cast<int>(g.K);
     kw = g.kw;
     W = g.W;
+    C = g.C;
     tap = g.tapW != 0;
     inner = tap ? g.C : g.kh * g.kw;
     HW4 = static_cast<uint32_t>(g.H) * static_cast<uint32_t>(g.W) * 4u;
@@ -86,7 +87,7 @@ struct GatherCols {
         const int ky = div_by(t, div.kw), kx = t - ky * kw;
         const bool ok = k < K && (yMask & (1u << (ky & 31))) && (xMask & (1u << kx));
         reg[j][e] = buf_ld1s(rsrc, sel_off(ok, colOff + static_cast<uint32_t>(ky * W + kx) * 4u),
-                             static_cast<uint32_t>(c) * HW4);
+                             static_cast<uint32_t>(min(c, C - 1)) * HW4);  // c past K: kOOB
       }
   }
   __device__ inline f32x4 quad(int u) const { return f32x4{reg[u][0], reg[u][1], reg[u][2], reg[u][3]}; }

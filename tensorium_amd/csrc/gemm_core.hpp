@@ -46,6 +46,9 @@ typedef __attribute__((address_space(3))) f32x4 lds_f4;
 
 constexpr int kPad = 4;                 // LDS row padding (floats)
 constexpr uint32_t kOOB = 0x80000000u;  // buffer offset beyond every range: reads 0
+// A scalar offset is added to kOOB too and must stay below 2^31, or the sum
+// passes 2^32 and names a place inside the buffer again: a row or k past the
+// operand's end takes the last one's (min below, wave-uniform).
 constexpr int64_t kMaxBufBytes = 0x7FFFFFF0;  // largest operand a buffer resource spans
 
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int PF_ = 2, int OCC_ = 1>

@@ -85,7 +85,7 @@ struct RowsTailMN {
   __device__ inline void load(int64_t k0) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t so = static_cast<uint32_t>(static_cast<int>(k0) + e) * ld4;
+      const uint32_t so = static_cast<uint32_t>(min(static_cast<int>(k0) + e, K - 1)) * ld4;  // kOOB
 #pragma unroll
       for (int j = 0; j < NQ; ++j) {
         const uint32_t vo = sel_off(static_cast<int>(k0) + k4[j] + e < K, voff[j]);

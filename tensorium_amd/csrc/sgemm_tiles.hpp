@@ -49,10 +49,11 @@ __device__ inline void sgemm_store(const SgemmArgs& a, int64_t bz, int64_t m0, i
     const int64_t n = n0w + j * 32 + (lane & 31);
     vo[j] = sel_off(n < a.N, static_cast<uint32_t>(rowBase) * ldc4 + static_cast<uint32_t>(n) * 4u);
   }
-  auto rowOff = [&](int i, int r) { return static_cast<uint32_t>(i * 32 + 8 * (r >> 2) + (r & 3)); };
-  auto off = [&](int i, int j, int r) {
-    return allRows || rowBase + static_cast<int>(rowOff(i, r)) < a.M ? vo[j] : kOOB;
-  };
+  auto rowOk = [&](int i, int r) { return allRows || rowBase + i * 32 + 8 * (r >> 2) + (r & 3) < a.M; };
+  auto off = [&](int i, int j, int r) { return rowOk(i, r) ? vo[j] : kOOB; };
+  // the row of a scalar offset: none past the last (kOOB)
+  const int lastRow = __builtin_amdgcn_readfirstlane(max(static_cast<int>(a.M - 1 - m0w), 0));
+  auto rowOff = [&](int i, int r) { return static_cast<uint32_t>(min(i * 32 + 8 * (r >> 2) + (r & 3), lastRow)); };
   const float alpha = a.alpha, beta = a.beta;
   if (a.splits > 1) {
     const __amdgpu_buffer_rsrc_t pR = make_rsrc(a.part + blockIdx.z * a.M * a.N, a.M * a.N * 4);
@@ -66,8 +67,7 @@ __device__ inline void sgemm_store(const SgemmArgs& a, int64_t bz, int64_t m0, i
             sel_off(n < a.N, static_cast<uint32_t>(rowBase) * n4 + static_cast<uint32_t>(n) * 4u);
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          conv::buf_st1s(pR, acc[i][j][r],
-                         allRows || rowBase + static_cast<int>(rowOff(i, r)) < a.M ? pv : kOOB, rowOff(i, r) * n4);
+          conv::buf_st1s(pR, acc[i][j][r], rowOk(i, r) ? pv : kOOB, rowOff(i, r) * n4);
       }
     return;
   }
