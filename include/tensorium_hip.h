@@ -115,7 +115,11 @@ int32_t tnh_stream_destroy(void *stream);
 /* ---- GEMM ------------------------------------------------------------- */
 /* TNNCuda.gemm (nncuda.pas:624) / cblas_sgemm (ntensors.pas:2231):
  * C = alpha*op(A)*op(B) + beta*C, all four NN/NT/TN/TT variants.
- * beta = 0 overwrites C without reading it (BLAS semantics). */
+ * beta = 0 overwrites C without reading it (BLAS semantics).  Large products,
+ * here and in the convolutions and weight gradients, are formed on the bf16
+ * matrix cores from three exact parts of every float; a tile with an infinity
+ * or NaN, a value past 2^103 or a sum past 2^80 is computed in fp32, more
+ * slowly. */
 int32_t tnh_sgemm(int32_t transA, int32_t transB, int64_t M, int64_t N,
                   int64_t K, float alpha, const float *A, int64_t aOff,
                   int64_t lda, const float *B, int64_t bOff, int64_t ldb,
