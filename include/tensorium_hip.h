@@ -880,7 +880,9 @@ int32_t tnh_conv2d_wgrad(int64_t batch, int64_t C, int64_t H, int64_t W,
  * alpha = beta = 1.  pieces NULL: only *nPieces is set (the count depends
  * on the geometry and the device's CU count, not on the data).  Refused
  * (TNH_ERR_UNSUPPORTED) for fewer than 8192 weights cut into several pieces,
- * which tnh_conv2d_wgrad sums a wave per weight in another order.  The pieces
+ * which tnh_conv2d_wgrad sums a wave per weight in another order; up to 480
+ * output pixels in all they are one piece, which tnh_conv2d_wgrad may cut (the
+ * last bits then differ).  The pieces
  * live in the caller's memory, so several layers' products can wait for one
  * update. */
 int32_t tnh_conv2d_wgrad_pieces(int64_t batch, int64_t C, int64_t H, int64_t W,

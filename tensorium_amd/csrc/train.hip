@@ -1010,9 +1010,6 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(WgradArgs a) {
   }
 }
 
-// weight gradients of fewer elements sum their pieces a wave per element
-constexpr int64_t kWaveReduceBelow = 8192;
-
 int launch_wgrad_reduce(const WgradArgs& a, hipStream_t s) {
   if (a.splits > 1 && !a.rawPieces) {
     // few outputs: a wave per output element spreads the splits over its

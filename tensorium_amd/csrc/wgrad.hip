@@ -229,20 +229,63 @@ using W64x128 = conv::LeanCfg<64, 128, 32, 2, 2, 2>;
 using W128x64 = conv::LeanCfg<128, 64, 32, 2, 2, 2>;
 using W64 = conv::LeanCfg<64, 64, 32, 2, 2, 3>;
 
+// What a tile costs a panel, in us: with one workgroup on its CU and, for each
+// of several, where the CU is busy.
+struct TileCost {
+  int rows, cols;
+  float alone, busy;
+};
+constexpr TileCost kTiles[] = {
+    {128, 128, 1.55f, 1.55f}, {64, 128, 1.5f, 1.05f}, {128, 64, 1.3f, 1.05f}, {64, 64, 0.9f, 0.6f}};
+
+struct Plan {
+  int tile, splits;
+  int64_t chunk;  // panels per split
+};
+
+// The tile and the split of the reduction axis, chosen together: a 128x128
+// tile reads the fewest bytes per product, but a short axis then leaves most
+// CUs without work, and each split costs its M*N floats written and read.
+// Every tile is tried whole and with the splits that give one, two and three
+// workgroups a CU, at least two panels each, and the least estimate taken.  The
+// constants are fitted to 1300 timings of 39 products (M 17 to 1024, N 27 to
+// 4608, 7 to 10816 panels), which they give within 10% in the mean; the choice
+// is within 5% of the best of each in the mean, 17% at most.  Layers of
+// 3 -> 32, 32 -> 64 and 64 -> 128 channels on 32x32, 16x16 and 8x8 pixels (us;
+// first the widest tile that fits with at least eight panels a split, then
+// this rule): batch 8 15.0, 19.7, 20.0 and 10.1, 10.5, 9.8; batch 32 16.0,
+// 21.6, 21.1 and 13.5, 15.8, 14.5; batch 128 22.4, 33.7, 26.4 and 22.3, 29.1,
+// 24.9.
+Plan plan(int64_t M, int64_t N, int64_t panels, int64_t cus) {
+  Plan best{0, 1, panels};
+  float least = 0.f;
+  for (int t = 0; t < 4; ++t) {
+    const TileCost& c = kTiles[t];
+    const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols);
+    for (int64_t n = 0; n <= 3; ++n) {
+      int64_t splits = std::max<int64_t>(1, std::min<int64_t>({n * cus / tiles, panels / 2, 1024}));
+      const int64_t chunk = (panels + splits - 1) / splits;
+      splits = (panels + chunk - 1) / chunk;  // no empty split
+      const int64_t perCU = (tiles * splits + cus - 1) / cus;
+      float us = static_cast<float>(chunk) * std::max(c.alone, static_cast<float>(perCU) * c.busy);
+      if (splits > 1)  // the reduction: a wave an element, or a thread
+        us += 2.f + static_cast<float>(splits) *
+                        (M * N < kWaveReduceBelow ? 0.006f : static_cast<float>(M * N) * 2.5e-6f);
+      if ((t == 0 && n == 0) || us < least) least = us, best = {t, static_cast<int>(splits), chunk};
+    }
+  }
+  return best;
+}
+
 template <class Cfg>
-int run(Context* cx, WgradArgs* a, const ColGeom* geom, const QuadAxis& ax, int perCU) {
+int run(Context* cx, WgradArgs* a, const ColGeom* geom, const QuadAxis& ax, const Plan& pl) {
   const int64_t tm = (a->M + Cfg::BM - 1) / Cfg::BM, tn = (a->N + Cfg::BN - 1) / Cfg::BN;
   if (tm * tn > INT32_MAX) return fail(TNH_ERR_UNSUPPORTED, "conv2d_wgrad: grid too large");
   a->tilesM = static_cast<int>(tm);
   a->tilesN = static_cast<int>(tn);
-  // one round of resident workgroups, at least eight panels each (a split
-  // costs its first panels' latency and M*N floats written and read)
   const int64_t panels = (ax.quads + 7) / 8;
-  int64_t splits = static_cast<int64_t>(perCU) * cx->cu_count / (tm * tn);
-  splits = std::max<int64_t>(1, std::min<int64_t>({splits, panels / 8, 1024}));
-  const int64_t chunk = (panels + splits - 1) / splits;
-  a->kChunk = chunk * 32;
-  a->splits = static_cast<int>((panels + chunk - 1) / chunk);
+  a->kChunk = pl.chunk * 32;
+  a->splits = pl.splits;
   if (a->rawPieces && !a->part) return TNH_OK;
   if (a->splits > 1 && !a->rawPieces) {
     a->part = static_cast<float*>(workspace(cx, static_cast<size_t>(a->splits) * a->M * a->N * 4));
@@ -288,12 +331,16 @@ int wgrad_any(Context* cx, WgradArgs* a, const ColGeom* geom) {
     *a = b;
     geom = nullptr;
   }
-  // 128x128 tiles read the fewest bytes per product; narrower ones where half
-  // a tile would be padding
-  if (a->M > 64 && a->N > 64) return run<W128>(cx, a, geom, ax, 1);
-  if (a->N > 64) return run<W64x128>(cx, a, geom, ax, 2);
-  if (a->M > 64) return run<W128x64>(cx, a, geom, ax, 2);
-  return run<W64>(cx, a, geom, ax, 3);
+  const int64_t panels = (ax.quads + 7) / 8;
+  Plan pl = plan(a->M, a->N, panels, cx->cu_count);
+  // the update pass takes few weights in one piece only
+  if (a->rawPieces && a->M * a->N < kWaveReduceBelow && panels < 16) pl = {3, 1, panels};
+  switch (pl.tile) {
+    case 0: return run<W128>(cx, a, geom, ax, pl);
+    case 1: return run<W64x128>(cx, a, geom, ax, pl);
+    case 2: return run<W128x64>(cx, a, geom, ax, pl);
+    default: return run<W64>(cx, a, geom, ax, pl);
+  }
 }
 
 }  // namespace tnh

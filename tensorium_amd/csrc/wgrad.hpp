@@ -16,6 +16,9 @@ struct WgradArgs {
   int rawPieces;  // store every split's raw sums in part, no reduction (also one split)
 };
 
+// weight gradients of fewer elements sum their pieces a wave per element
+constexpr int64_t kWaveReduceBelow = 8192;
+
 // A convolution's input as the column operand: [C][H][W] images, kernel, stride, padding, dilation.
 struct ColGeom {
   int64_t xBatchStride, xBytes;

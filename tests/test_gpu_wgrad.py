@@ -89,3 +89,34 @@ def test_infinite_input_outside_the_rows(hip):
     ref = np.matmul(delta.astype(np.float64), col.astype(np.float64).transpose(0, 2, 1)).sum(0)
     assert np.isinf(ref).any() and np.isfinite(ref).any()
     assert np.array_equal(dW.cpu().numpy(), ref.astype(np.float32))
+
+
+@pytest.mark.parametrize("B,C,H,F", [(8, 32, 16, 64), (8, 64, 8, 128), (32, 64, 8, 128), (128, 32, 16, 64), (128, 64, 8, 128)])
+def test_short_axes_fill_the_gpu(hip, B, C, H, F):
+    """A quarter of the workgroups that 64x64 tiles of two panels of 32 pixels
+    would give, or one a CU: neither large tiles nor long splits leave the GPU
+    idle."""
+    print(f"[case] wgrad pieces B{B} C{C} {H}x{H} F{F}", flush=True)
+    K, panels = C * 9, B * H * H // 32
+    x, d = torch.zeros(B, C, H, H, device="cuda"), torch.zeros(B, F, H, H, device="cuda")
+    n = hip.convWeightGradientPieces(B, C, H, H, F, 3, 3, 1, 1, 1, 1, 1, 1, x, C * H * H, d, F * H * H)
+    tiles = -(-F // 64) * -(-K // 64)
+    assert n * tiles >= min(tiles * panels // 8, 256)
+
+
+def test_few_weights_on_a_short_axis_are_one_piece(hip):
+    """Fewer than 8192 weights: one piece up to 15 panels of 32 pixels, refused above."""
+    print("[case] wgrad pieces few weights", flush=True)
+    C, H, F = 3, 8, 32
+    for B in (1, 4, 7):
+        x, d = torch.ones(B, C, H, H, device="cuda"), torch.ones(B, F, H, H, device="cuda")
+        pieces = torch.zeros(F * C * 9, device="cuda")
+        torch.cuda.synchronize()
+        assert hip.convWeightGradientPieces(B, C, H, H, F, 3, 3, 1, 1, 1, 1, 1, 1, x, C * H * H, d, F * H * H, pieces,
+                                            F * C * 9) == 1
+        hip.finish()
+        col, _, _ = im2col(np.ones((B, C, H, H), np.float32), 3, 3, 1, 1, 1, 1, 1, 1)
+        assert np.array_equal(pieces.cpu().numpy().reshape(F, C * 9), np.tile(col.sum((0, 2)), (F, 1)))
+    x, d = torch.ones(8, C, H, H, device="cuda"), torch.ones(8, F, H, H, device="cuda")
+    with pytest.raises(Exception, match="sum their pieces a wave each"):
+        hip.convWeightGradientPieces(8, C, H, H, F, 3, 3, 1, 1, 1, 1, 1, 1, x, C * H * H, d, F * H * H)
