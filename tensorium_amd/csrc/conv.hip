@@ -711,8 +711,13 @@ int conv_dispatch(Context* cx, ConvArgs& a, int mode, bool va, bool vb, bool sma
     const CfgInfo& ci = kCfgs[c];
     const int64_t tiles = tilesOf(ci);
     if (tiles >= 2 * cus || det) continue;
+    // at least four panels a split; two for the gather tiles, which wait on a
+    // panel's single loads (1.6 us) longer than a split costs (5x5, 65 -> 35
+    // channels, 15x15: 4 and 8 splits 23.2 and 16.3 us, the fp32 tiles that
+    // they replaced 15.2)
+    const int64_t least = ci.kind == kGather ? 2 : 4;
     for (int sp : {2, 4, 8, 16})
-      if (tiles * sp <= 8 * cus && K >= static_cast<int64_t>(sp) * ci.BK * 4)
+      if (tiles * sp <= 8 * cus && K >= sp * ci.BK * least)
         cands.push_back(nhwc ? Cand{c, 1, sp, 2} : Cand{c, sp, 0, 0});
   }
   auto unitOf = [&](const Cand& c) -> int64_t {

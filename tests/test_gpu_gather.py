@@ -108,3 +108,22 @@ def test_gather_infinite_input_and_weight_rows(hip, cfg):
     hip.finish()
     assert np.isinf(ref[0, 3]).all() and np.isfinite(ref[0, 2]).any()
     assert np.array_equal(out.cpu().numpy(), ref.astype(np.float32))
+
+
+@pytest.mark.parametrize("cfg", GATHER)
+@pytest.mark.parametrize("B,C,H,W,F,k,s,splits", [(1, 65, 15, 15, 35, 5, 1, 16), (2, 32, 13, 10, 32, 5, 2, 8),
+                                                  (1, 7, 13, 13, 16, 7, 1, 4)])
+def test_gather_splits_of_a_few_panels(hip, cfg, B, C, H, W, F, k, s, splits):
+    """The K splits that small layers are timed with: two to four panels of 32 each, a remainder in the last."""
+    print(f"[case] conv gather splits cfg {cfg} C {C} k {k} splits {splits}", flush=True)
+    x, w = np.round(synth.normal(1220, (B, C, H, W), 2.0)), np.round(synth.normal(1221, (F, C, k, k), 1.5))
+    ref = conv64(x, w, s, k // 2, k // 2).astype(np.float32)
+    dx, dw, out = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), torch.zeros(ref.shape, device="cuda")
+    torch.cuda.synchronize()
+    hip.setConvAutotune(True, cfg + CONV_SPLIT_UNIT * splits)
+    try:
+        hip.conv2dForward(B, C, H, W, F, k, s, k // 2, dx, 0, dw, None, 4, out, 0)
+    finally:
+        hip.setConvAutotune(True, -1)
+    hip.finish()
+    assert np.array_equal(out.cpu().numpy(), ref)
