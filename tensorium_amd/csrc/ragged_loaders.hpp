@@ -67,19 +67,26 @@ struct RowsTailMN {
   int ldsOff[NQ][CPT], k4[NQ], K;
   Reg reg[NQ][4];
 
-  __device__ inline void init(const float* p, int64_t bytes, int64_t ld, int64_t rows, int64_t r0, int tid) {
+  // rowOff(row): as SplitRowsMN's
+  template <class F>
+  __device__ inline void init_rows(const float* p, int64_t bytes, int64_t ld, int tid, F&& rowOff) {
     rsrc = make_rsrc(p, bytes);
     ld4 = static_cast<uint32_t>(ld) * 4u;
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
       const int u = tid + j * NT;
       const int row = CPT * ((u & 3) | (u >> 5 << 2)), kq = (u >> 2) & 7;
-      voff[j] = r0 + row < rows ? static_cast<uint32_t>((r0 + row + 4 * kq * ld) * 4) : kOOB;
+      const uint32_t o = rowOff(row);
+      voff[j] = o != kOOB ? o + static_cast<uint32_t>(4 * kq) * ld4 : kOOB;  // wraps only past K
       k4[j] = 4 * kq;
 #pragma unroll
       for (int c = 0; c < CPT; ++c) ldsOff[j][c] = L::chunk(row + c, kq);
     }
     K = 0;
+  }
+  __device__ inline void init(const float* p, int64_t bytes, int64_t ld, int64_t rows, int64_t r0, int tid) {
+    init_rows(p, bytes, ld, tid,
+              [&](int row) { return r0 + row < rows ? static_cast<uint32_t>((r0 + row) * 4) : kOOB; });
   }
   __device__ inline void klimit(int64_t k) { K = static_cast<int>(k); }
   __device__ inline void load(int64_t k0) {

@@ -24,6 +24,11 @@ SHAPES = [
     (3, 48, 8, 17, 100, 3, 3, 1, 1, 1),
     (1, 70, 13, 13, 64, 3, 3, 1, 1, 1),
     (2, 3, 4, 4, 40, 5, 5, 1, 4, 4),
+    # 1x1 over whole planes, pixels a multiple of 4: rows of pixels in units of 2 and 4
+    (2, 13, 6, 10, 129, 1, 1, 1, 0, 0),
+    (3, 70, 7, 8, 65, 1, 1, 1, 0, 0),
+    (1, 33, 1, 4, 20, 1, 1, 1, 0, 0),
+    (5, 1, 2, 2, 3, 1, 1, 1, 0, 0),
 ]
 
 
