@@ -143,6 +143,8 @@ int32_t tnh_sgemm_strided_batched(int32_t transA, int32_t transB, int64_t M,
  * library's choice), 10..12 the 128x128 / 64x128 / 64x64 tiles for any
  * operands (C within 2 GiB), 6..8 the wave-split 32x32 (4 or 8 waves) and 32x64 tiles
  * (K split over the waves of one workgroup; the lean tiles' requirements);
+ * plus 64 times a number of K splits (0 or 1: none; up to 64) for tiles 2..5
+ * and 10..12 and one batch item, other tiles and batches are then refused;
  * -1 lets the library choose.  The whole-K lean and any-operand
  * configurations sum k in the same order; K splits of the under-filled ones
  * (timed, never in the deterministic mode) sum their partials in order; the

@@ -378,6 +378,8 @@ RaggedInfo split_tile(int cfg) {
 struct SgemmPick {
   int cfg, splits;
 };
+constexpr int kSplitUnit = 64;   // a forced configuration: tile + kSplitUnit * splits
+constexpr int kMostSplits = 64;
 
 // part: the partials of pick.splits > 1 splits (nullptr: whole K).
 int launch_sgemm(const SgemmPick& pick, const SgemmArgs& a0, int64_t batch, bool ta, bool tb, bool va, bool vb,
@@ -483,7 +485,13 @@ int sgemm_impl(int32_t transA, int32_t transB, int64_t M, int64_t N, int64_t K, 
     std::lock_guard<std::mutex> lk(g_sgemm_mu);
     auto it = g_sgemm_tuned.find(key);
     if (g_sgemm_forced >= 0) {
-      if (g_sgemm_forced < kL128x128 || (g_sgemm_forced >= kRagged ? small : lean)) cfg = g_sgemm_forced;
+      const int c = g_sgemm_forced % kSplitUnit, sp = g_sgemm_forced / kSplitUnit;
+      if (c < kL128x128 || (c >= kRagged ? small : lean)) {
+        if (sp > 1 && (!split_tile(c).rows || batch != 1 || M * N * 4 > kMaxBufBytes))
+          return fail(TNH_ERR_UNSUPPORTED, "sgemm: forced K split of a tile or batch that does not split");
+        cfg = c;
+        splits = std::max(1, sp);
+      }
     } else if (deterministic()) {
       // the untuned choice from the shape alone
     } else if (it != g_sgemm_tuned.end()) {
@@ -502,7 +510,7 @@ int sgemm_impl(int32_t transA, int32_t transB, int64_t M, int64_t N, int64_t K, 
     if (!t.rows || batch != 1 || M * N * 4 > kMaxBufBytes) return 1;
     const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
     const int64_t sp = static_cast<int64_t>(t.perCU) * cx->cu_count / tiles;
-    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({sp, (K + 31) / 32 / 8, 64})));
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({sp, (K + 31) / 32 / 8, kMostSplits})));
   };
   auto partOf = [&](int sp) -> float* {
     return sp > 1 ? static_cast<float*>(workspace(cx, static_cast<size_t>(sp) * M * N * 4)) : nullptr;
@@ -566,7 +574,9 @@ int sgemm_impl(int32_t transA, int32_t transB, int64_t M, int64_t N, int64_t K, 
 }  // namespace tnh
 
 extern "C" int32_t tnh_sgemm_set_autotune(int32_t enable, int32_t forcedConfig) {
-  TNH_ARG(forcedConfig >= -1 && forcedConfig < tnh::kNumSgemmCfg, "sgemm_set_autotune: config %d", forcedConfig);
+  TNH_ARG(forcedConfig >= -1 && (forcedConfig < 0 || forcedConfig % tnh::kSplitUnit < tnh::kNumSgemmCfg) &&
+              forcedConfig / tnh::kSplitUnit <= tnh::kMostSplits,
+          "sgemm_set_autotune: config %d", forcedConfig);
   std::lock_guard<std::mutex> lk(tnh::g_sgemm_mu);
   tnh::g_sgemm_autotune = enable != 0;
   tnh::g_sgemm_forced = forcedConfig;

@@ -51,6 +51,7 @@ CONV_TAIL_SLOT_BASE = 32
 # SGEMM tile configurations (tnh_sgemm_set_autotune): 0, 1 general, 2..5 and 9
 # lean, 6..8 wave-split, 10..12 any operands
 NUM_SGEMM_CFGS = 13
+SGEMM_SPLIT_UNIT = 64  # a forced id is tile + SGEMM_SPLIT_UNIT * K splits (tiles 2..5 and 10..12)
 
 i32, i64, f32, vp = C.c_int32, C.c_int64, C.c_float, C.c_void_p
 
