@@ -1,30 +1,15 @@
-// Lean implicit-GEMM convolution on fp32 MFMA (gfx950).
-//
-// The fastest conv kernel family of the library.  What makes it lean:
+// Operand loaders of the lean tiles and of the wave-split tiles (conv_wsplit),
+// their fp32 LDS panels and the fp32 fragments.  The lean tiles' loop is
+// split_loop.hpp's, which takes the loaders with its own panels.
 //   * Both operand panels are k-contiguous in LDS with their 16-byte chunks
-//     XOR-swizzled by row % 8: every LDS access is a conflict-free 16-byte
+//     XOR-swizzled: every LDS access is a conflict-free 16-byte
 //     ds_read/ds_write_b128 and no padding is needed.  The B gather writes 4
-//     consecutive k of one output column per 16-byte store.
+//     consecutive k of one output column per store.
 //   * Per-lane global offsets are fixed for the whole K loop; what varies
 //     along K is wave-uniform and rides in the buffer instruction's scalar
 //     offset.  The 3x3 padding test is a per-lane 9-bit tap mask computed
 //     once, so a K panel costs a few vector ALU operations instead of two per
 //     load.
-//   * Schedule of panel p (two LDS stages; the loaders' registers hold panel
-//     p+1; the fragments of chunk 0 of panel p are in registers):
-//       chunks 0 .. KCH-2: read the fragments of chunk c+1, then the MFMAs of
-//         chunk c; during chunk 0 the registers of panel p+1 go to the other
-//         stage and the global loads of panel p+2 are issued;
-//       barrier (every wave stored panel p+1 and read all of panel p);
-//       read the fragments of chunk 0 of panel p+1, then the MFMAs of chunk
-//       KCH-1 of panel p.
-//     The other stage held panel p-1, whose last reads precede the previous
-//     barrier, so overwriting it during panel p is safe; panel p+1 is read
-//     only after this panel's barrier.  A wave reaches the barrier with the
-//     last chunk's MFMAs still to issue, and the first fragment reads of the
-//     next panel hide behind them.  The panel loop is unrolled over the two
-//     stages (LDS addresses are per-lane constants plus immediates) and the
-//     last panels are peeled, so the steady-state body is one basic block.
 //
 // Requirements (checked by the host): K % BK == 0 (tap-major 3x3 with
 // C % BK == 0, or 1x1 stride 1 with C % BK == 0), 16-byte weight rows, and
@@ -43,7 +28,7 @@ struct LeanCfg {
   static constexpr int FM = WTM / 32, FN = WTN / 32;
   static constexpr int KCH = BK / 16;
   static_assert(FM >= 1 && FN >= 1 && WTM % 32 == 0 && WTN % 32 == 0, "tile");
-  static_assert(BK % 32 == 0 && KCH % 2 == 0, "BK: 32 or 64");
+  static_assert(BK == 32, "panel depth");
 };
 
 // k-contiguous panel [ROWS][BK] (floats) whose 16-byte chunks are
@@ -52,15 +37,14 @@ struct LeanCfg {
 // lanes at a time, so 16 consecutive rows at one logical chunk must land in
 // 16 different 16-byte bank groups.  A 32-float row is half a bank line: the
 // row parity picks the half and swz(r) = (r / 2) % 8 spreads each half's 8
-// rows over its 8 groups.  A 64-float row spans all 64 banks: swz(r) =
-// r % 16.  One row's chunks, and two consecutive rows' chunks, are always
-// distinct groups too (the row-wise stores of the loaders).
+// rows over its 8 groups.  One row's chunks, and two consecutive rows' chunks,
+// are always distinct groups too (the row-wise stores of the loaders).
 template <int ROWS, int BK>
 struct SwzPanel {
   static constexpr int SIZE = ROWS * BK;
   static constexpr int STRIDE = BK;  // floats per row
-  static_assert(BK == 32 || BK == 64, "panel depth");
-  __device__ static inline int swz(int row) { return BK == 32 ? (row >> 1) & 7 : row & 15; }
+  static_assert(BK == 32, "panel depth");
+  __device__ static inline int swz(int row) { return (row >> 1) & 7; }
   __device__ static inline int chunk(int row, int q) { return row * BK + 4 * (q ^ swz(row)); }
   // four consecutive k of a row to the place chunk() names
   __device__ static inline void put(lds_t* p, f32x4 v) { *reinterpret_cast<lds_f4*>(p) = v; }
@@ -130,58 +114,39 @@ using LeanA = LeanRowsK<Cfg::BM, Cfg::BK, Cfg::NT>;
 
 // Row-contiguous operand: element (row r, k) at (r0 + r) + k * ld floats
 // (rows >= `rows` read 0): the GEMM operands A (transposed) and B (not
-// transposed).  VEC (ld % 4 == 0, rows % 4 == 0, 16-byte aligned base):
-// thread t owns rows 4 * (t % (ROWS/4)) .. +3 and k-quads t / (ROWS/4) + j *
-// QSTEP; it loads a 4 (k) x 4 (row) block with four 16-byte loads and stores
-// its transpose, one 16-byte LDS write per row.  Scalar: one row per thread,
-// 4 loads ld floats apart per k-quad.
-template <int ROWS, int BK_, int NT_, bool VEC, template <int, int> class Panel = SwzPanel>
+// transposed) in fp32.  Thread t owns row t % ROWS and the k-quads t / ROWS +
+// j * QSTEP, four loads ld floats apart each.
+template <int ROWS, int BK_, int NT_>
 struct LeanRowsMN {
   static constexpr int BK = BK_, NT = NT_;
-  static constexpr int CPT = VEC ? 4 : 1;
-  static constexpr int TPR = ROWS / CPT;
-  static constexpr int QSTEP = NT / TPR, NQ = (BK / 4) / QSTEP;
-  using L = Panel<ROWS, BK>;
+  static constexpr int QSTEP = NT / ROWS, NQ = (BK / 4) / QSTEP;
+  using L = SwzPanel<ROWS, BK>;
   static constexpr int SIZE = L::SIZE;
-  static_assert(NT % TPR == 0 && (BK / 4) % QSTEP == 0 && NQ >= 1, "LeanRowsMN split");
-  using Reg = typename std::conditional<VEC, f32x4, float>::type;
+  static_assert(NT % ROWS == 0 && (BK / 4) % QSTEP == 0 && NQ >= 1, "LeanRowsMN split");
   __amdgpu_buffer_rsrc_t rsrc;
   uint32_t voff, ld4;
-  int ldsOff[NQ][CPT];
-  Reg reg[NQ][4];
+  int ldsOff[NQ];
+  float reg[NQ][4];
 
   __device__ inline void init(const float* p, int64_t bytes, int64_t ld, int64_t rows, int64_t r0, int tid) {
     rsrc = make_rsrc(p, bytes);
     ld4 = static_cast<uint32_t>(ld) * 4u;
-    const int row = (tid % TPR) * CPT, q0 = tid / TPR;
+    const int row = tid % ROWS, q0 = tid / ROWS;
     const int64_t gr = r0 + row;
     voff = sel_off(gr < rows, static_cast<uint32_t>((gr + 4 * q0 * ld) * 4));
 #pragma unroll
-    for (int j = 0; j < NQ; ++j)
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) ldsOff[j][c] = L::chunk(row + c, q0 + j * QSTEP);
+    for (int j = 0; j < NQ; ++j) ldsOff[j] = L::chunk(row, q0 + j * QSTEP);
   }
   __device__ inline void load(int64_t k0) {
 #pragma unroll
     for (int j = 0; j < NQ; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t so = static_cast<uint32_t>(static_cast<int>(k0) + 4 * j * QSTEP + e) * ld4;
-        if constexpr (VEC)
-          reg[j][e] = buf_ld4s(rsrc, voff, so);
-        else
-          reg[j][e] = buf_ld1s(rsrc, voff, so);
-      }
+      for (int e = 0; e < 4; ++e)
+        reg[j][e] = buf_ld1s(rsrc, voff, static_cast<uint32_t>(static_cast<int>(k0) + 4 * j * QSTEP + e) * ld4);
   }
-  static constexpr int QUADS = NQ * CPT;
-  __device__ inline f32x4 quad(int u) const {
-    const int j = u / CPT, c = u % CPT;
-    if constexpr (VEC)
-      return f32x4{reg[j][0][c], reg[j][1][c], reg[j][2][c], reg[j][3][c]};
-    else
-      return f32x4{reg[j][0], reg[j][1], reg[j][2], reg[j][3]};
-  }
-  __device__ inline int off(int u) const { return ldsOff[u / CPT][u % CPT]; }
+  static constexpr int QUADS = NQ;
+  __device__ inline f32x4 quad(int u) const { return f32x4{reg[u][0], reg[u][1], reg[u][2], reg[u][3]}; }
+  __device__ inline int off(int u) const { return ldsOff[u]; }
   __device__ inline void store(lds_t* stage) const { store_quads(*this, stage); }
 };
 

@@ -73,7 +73,7 @@ struct Op {  // k contiguous
 template <class Cfg, int ROWS>
 struct Op<Cfg, ROWS, false> {  // rows contiguous
   using split = conv::SplitRowsMN<ROWS, Cfg::NT>;
-  using plain = conv::LeanRowsMN<ROWS, Cfg::BK, Cfg::NT, false>;
+  using plain = conv::LeanRowsMN<ROWS, Cfg::BK, Cfg::NT>;
 };
 
 template <class Cfg, bool TA, bool TB>
