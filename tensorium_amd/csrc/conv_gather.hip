@@ -96,7 +96,7 @@ struct GatherCols {
 };
 
 // A 1x1 window over every pixel: the columns are the channels' own rows of
-// pixels, in RowsTailMN's units (OHW % 4 == 0: none crosses an image's end).
+// pixels, in RowsTailMN's units, none of which may cross an image's end.
 // Loaded element by element such a layer, which multiplies little, waited on
 // its loads: 200 -> 300 channels, 26x26, batch 4 15.2 -> 10.6 us, 48 -> 100,
 // 60x60, batch 8 12.1 -> 9.5 (the fp32 tiles before 12.8 and 14.7).
@@ -113,28 +113,18 @@ struct PixelCols : RowsTailMN<Cfg::BN, Cfg::NT, Panel> {
   }
 };
 
-template <class Cfg, bool PIX, template <int, int> class P>
-struct GatherB {
-  using type = GatherCols<Cfg, P>;
-};
-template <class Cfg, template <int, int> class P>
-struct GatherB<Cfg, true, P> {
-  using type = PixelCols<Cfg, P>;
-};
-
-template <class Cfg, bool PIX>
-__global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void conv_gather_kernel(ConvArgs a, GatherDiv d) {
+// One tile, its columns loaded by BL (in fp32: BF).  A function that takes the
+// arguments by reference: with the same code in the kernel, on its own copy of
+// them, the compiler spilled (64x64 over rows of pixels 168 registers and 40
+// bytes of scratch, here 124; 5x5, 48 -> 100, 57x75, batch 8 124.3 -> 120.3 us).
+// The SGEMM tiles, written so, use 40 registers less too and are 3 to 5% slower.
+template <class Cfg, class BL, class BF>
+__device__ inline void gather_tile(const ConvArgs& a, const GatherDiv& d, int64_t m0, int64_t n0, lds_t* lds, int* odd) {
+  f32x16 acc[Cfg::FM][Cfg::FN];
   using AL = RowsTailK<Cfg::BM, Cfg::NT, SplitPanel>;
   using AF = RowsTailK<Cfg::BM, Cfg::NT, SwzPanel>;
-  using BL = typename GatherB<Cfg, PIX, SplitPanel>::type;
-  using BF = typename GatherB<Cfg, PIX, SwzPanel>::type;
   using Loop = SplitLoop<Cfg, AL, BL>;
-  __shared__ __attribute__((aligned(16))) float smem[Loop::LDS_FLOATS];
-  __shared__ int odd;
-  lds_t* lds = (lds_t*)smem;
-  int tm, tn;
-  tile_coords(blockIdx.x, a.tilesM, a.tilesN, tm, tn);
-  const int64_t m0 = static_cast<int64_t>(tm) * Cfg::BM, n0 = static_cast<int64_t>(tn) * Cfg::BN;
+  static_assert(Loop::LDS_FLOATS == kSplitLds<Cfg>, "panels");
   auto init = [&](auto& al, auto& bl) {
     al.init(a.w, a.wBytes, a.g.K, a.F, m0, threadIdx.x);
     al.klimit(a.g.K);
@@ -145,9 +135,8 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void conv_gather_kernel(ConvArgs
   AL al;
   BL bl;
   init(al, bl);
-  f32x16 acc[Cfg::FM][Cfg::FN];
-  Loop::exec(al, bl, kBegin, nk, lds, &odd, acc);
-  if (!Loop::finite(acc, &odd)) {
+  Loop::exec(al, bl, kBegin, nk, lds, odd, acc);
+  if (!Loop::finite(acc, odd)) {
     AF af;
     BF bf;
     init(af, bf);
@@ -156,6 +145,30 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void conv_gather_kernel(ConvArgs
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
   conv_store_buf<Cfg::FM, Cfg::FN>(a, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, lane);
+}
+
+// How a kernel loads its columns: single elements, rows of pixels (1x1 windows,
+// images of whole units), or rows of pixels but single ones in the tiles that
+// hold an image's end (123 -> 37 channels, 187x187, batch 21 185 -> 155 us; 90
+// -> 142, 43x51, batch 23 38.3 -> 29.5).  The last needs more registers: not
+// for images of a few tiles (100 -> 255, 13x13, batch 16 11.0 -> 11.7), nor
+// where no unit crosses an image's end.
+enum GatherLoads { kElements, kPixels, kPixelsOrEnds };
+
+template <class Cfg, GatherLoads LOADS>
+__global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void conv_gather_kernel(ConvArgs a, GatherDiv d) {
+  __shared__ __attribute__((aligned(16))) float smem[kSplitLds<Cfg>];
+  __shared__ int odd;
+  lds_t* lds = (lds_t*)smem;
+  int tm, tn;
+  tile_coords(blockIdx.x, a.tilesM, a.tilesN, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * Cfg::BM, n0 = static_cast<int64_t>(tn) * Cfg::BN;
+  bool pixels = LOADS == kPixels;
+  if constexpr (LOADS == kPixelsOrEnds) pixels = n0 / a.g.OHW == (min(n0 + Cfg::BN, a.g.N) - 1) / a.g.OHW;
+  if constexpr (LOADS != kElements)
+    if (pixels) gather_tile<Cfg, PixelCols<Cfg, SplitPanel>, PixelCols<Cfg, SwzPanel>>(a, d, m0, n0, lds, &odd);
+  if constexpr (LOADS != kPixels)
+    if (!pixels) gather_tile<Cfg, GatherCols<Cfg, SplitPanel>, GatherCols<Cfg, SwzPanel>>(a, d, m0, n0, lds, &odd);
 }
 
 using G64 = LeanCfg<64, 64, 32, 2, 2, 3>;
@@ -174,10 +187,13 @@ int run(ConvArgs a, hipStream_t s) {
   const GatherDiv d{magic(a.g.tapW ? a.g.C : a.g.kh * a.g.kw), magic(a.g.kw)};
   const dim3 grid(static_cast<unsigned>(tm * tn), static_cast<unsigned>(a.splits));
   const ConvGeom& g = a.g;
-  if (g.kh == 1 && g.kw == 1 && g.sY == 1 && g.sX == 1 && g.pH == 0 && g.pW == 0 && g.OHW % 4 == 0)
-    hipLaunchKernelGGL((conv_gather_kernel<Cfg, true>), grid, dim3(Cfg::NT), 0, s, a, d);
+  const bool planes = g.kh == 1 && g.kw == 1 && g.sY == 1 && g.sX == 1 && g.pH == 0 && g.pW == 0;
+  if (planes && g.OHW % 4 == 0)
+    hipLaunchKernelGGL((conv_gather_kernel<Cfg, kPixels>), grid, dim3(Cfg::NT), 0, s, a, d);
+  else if (planes && g.OHW >= 8 * Cfg::BN)
+    hipLaunchKernelGGL((conv_gather_kernel<Cfg, kPixelsOrEnds>), grid, dim3(Cfg::NT), 0, s, a, d);
   else
-    hipLaunchKernelGGL((conv_gather_kernel<Cfg, false>), grid, dim3(Cfg::NT), 0, s, a, d);
+    hipLaunchKernelGGL((conv_gather_kernel<Cfg, kElements>), grid, dim3(Cfg::NT), 0, s, a, d);
   return launch_status("conv_gather_kernel");
 }
 

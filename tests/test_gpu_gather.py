@@ -29,6 +29,11 @@ SHAPES = [
     (3, 70, 7, 8, 65, 1, 1, 1, 0, 0),
     (1, 33, 1, 4, 20, 1, 1, 1, 0, 0),
     (5, 1, 2, 2, 3, 1, 1, 1, 0, 0),
+    # no multiple of 4: tiles with and without an image's end
+    (3, 33, 13, 15, 40, 1, 1, 1, 0, 0),
+    (2, 6, 1, 129, 33, 1, 1, 1, 0, 0),
+    (2, 35, 23, 29, 130, 1, 1, 1, 0, 0),
+    (3, 9, 37, 57, 40, 1, 1, 1, 0, 0),
 ]
 
 
