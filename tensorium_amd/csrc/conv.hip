@@ -682,7 +682,7 @@ int conv_dispatch(Context* cx, ConvArgs& a, int mode, bool va, bool vb, bool sma
   // NCHW: the gather tiles take what the lean tiles do not, and the fp32
   // LDS-staged tiles what neither does (an operand over 2 GiB; at 128 -> 256
   // channels, 52x52, batch 16 they take 247 us against the lean tiles' 148,
-  // at 5x5, 48 -> 100, 57x75, batch 8 206 against 118)
+  // at 5x5, 48 -> 100, 57x75, batch 8 206 against 120)
   bool lean = false, gather = false;
   for (int c = 0; c < kNumCfg && !nhwc; ++c)
     if (cfg_valid(c, mode, C, K, va, smallIO, nhwc)) {

@@ -504,7 +504,7 @@ int sgemm_impl(int32_t transA, int32_t transB, int64_t M, int64_t N, int64_t K, 
   }
   // K splits of a tile that leaves CUs idle: as many as fill the resident
   // workgroups, at least 8 panels each (255x1531x10817: 24 tiles of 128x128,
-  // 325 -> 55 us with K split)
+  // 325 -> 58 us with K split)
   auto splitsOf = [&](int c) -> int {
     const RaggedInfo t = split_tile(c);
     if (!t.rows || batch != 1 || M * N * 4 > kMaxBufBytes) return 1;
